@@ -101,3 +101,36 @@ def test_prefill_c4_shape():
     assert rel_l2(S, S_ref) <= 1e-4, rel_l2(S, S_ref)
     assert rel_l2(out, o_ref) <= 1e-2
     assert float((out - o_ref.float()).abs().max()) <= 2e-2
+
+
+# One round of workgroups decides the scan's slice width (16, 32 or 64 state
+# columns: up to 256, 512 and more column tiles b * h * d / 16 on 256 CUs); each
+# width at both head sizes, with whole and ragged last chunks.
+@pytest.mark.parametrize("B,T,H,d", [(1, 65, 3, 64), (1, 127, 2, 128), (5, 100, 16, 64),
+                                     (3, 64, 16, 128), (9, 70, 16, 64), (5, 129, 16, 128)])
+def test_prefill_slice_widths(B, T, H, d):
+    q, k, v, beta, gd, S0 = _inputs(B, T, H, d, 77 + T)
+    o_ref, S_ref = gdn_sequential(q.float(), k.float(), v.float(), beta, gd, S0)
+    out, S = _run(q, k, v, beta, gd, S0)
+    assert rel_l2(S, S_ref) <= 1e-4, rel_l2(S, S_ref)
+    assert float((out - o_ref).abs().max()) <= 2e-2
+    assert rel_l2(out, o_ref) <= 1e-2
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_prefill_unaligned_out_and_neighbours(d):
+    """An output that is only 2-byte aligned takes the narrow stores (same bits),
+    and a sequence's ragged last chunk reads nothing of the next sequence, whose
+    rows are NaN here."""
+    B, T, H = 2, 83, 2
+    q, k, v, beta, gd, S0 = _inputs(B, T, H, d, 5 + d)
+    out, S = _run(q, k, v, beta, gd, S0)
+    for t in (q, k, v, beta, gd):
+        t[1] = float("nan")
+    Sn = S0.clone().cuda()
+    buf = torch.zeros(B * T * H * d + 1, dtype=torch.bfloat16, device="cuda")
+    odd = buf[1:].view(B, T, H, d)
+    ops().gdn_prefill(q.cuda(), k.cuda(), v.cuda(), beta.cuda(), gd.cuda(), Sn, out=odd)
+    assert torch.equal(odd[0].float().cpu(), out[0])
+    assert torch.equal(Sn[0].cpu(), S[0])
+    assert float(buf[0]) == 0.0

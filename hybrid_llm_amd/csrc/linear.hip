@@ -623,8 +623,11 @@ int32_t dense_gemm_mfma(const uint16_t* x, const uint16_t* w, void* out, const f
 
 // Rows from which the dense projections switch from the weight-streaming
 // kernel (every weight byte read once per 64 rows, HBM-bound) to the MFMA
-// tiles (compute-bound); decode batches stay below it.
-constexpr int kDenseMfmaMinRows = 256;
+// tiles (compute-bound); decode batches stay below it.  us, bf16 out, packed
+// weights, streaming / tiles: 65 x 3072 x 1024 10.1 / 9.7, 65 x 1024 x 2048 15.1 /
+// 16.2, 96 x 1024 x 2048 17.4 / 16.4, 128 x 4112 x 1024 19.2 / 10.1, 255 x 1024 x
+// 1024 21.1 / 9.7, gated residual 30.2 / 13.0.
+constexpr int kDenseMfmaMinRows = 96;
 
 }  // namespace llmy
 

@@ -73,6 +73,39 @@ def test_linear_epilogues(M, N, K, epi, layout):
     assert torch.allclose(out.cpu(), expect, atol=1e-4, rtol=1e-4)
 
 
+# Rows from which the tiles take over, and one size per tile shape (128 x 128, 128
+# x 192, 128 x 256, 256 x 192, 256 x 256) with partial tiles in both directions.
+# Tolerances: fp32 sums of K products |x w| ~ 0.016 in another order (K 2^-24 K
+# 0.016 < 1e-5 at K = 512).
+@pytest.mark.parametrize("M,N,K", [(95, 1040, 512), (96, 1040, 512), (97, 48, 256),
+                                   (129, 3088, 256), (2030, 3040, 256), (2500, 3056, 256),
+                                   (4090, 3040, 256), (4001, 3984, 512), (2048, 4112, 256)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+def test_linear_tile_shapes(M, N, K, epi):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = _bf(torch.randn(M, K, generator=g, device="cuda"))
+    w = _bf(torch.randn(N, K, generator=g, device="cuda") * 0.02)
+    base = torch.randn(M, N, generator=g, device="cuda")
+    aux = torch.rand(M, N, generator=g, device="cuda")
+    ref = x.double() @ w.double().t()
+    expect = {0: ref, 1: ref, 2: base + ref, 3: base + ref * aux}[epi]
+    for layout in (0, 1):
+        wl = w if layout == 0 else ops().pack_weights(w)
+        # rows past M must stay untouched
+        buf = torch.full((M + 8, N), 7.0, dtype=torch.bfloat16 if epi == 0 else torch.float32,
+                         device="cuda")
+        if epi >= 2:
+            buf[:M] = base
+        ops().linear(x, wl, out=buf[:M], epilogue=epi, aux=aux if epi == 3 else None,
+                     layout=layout)
+        err = (buf[:M].double() - expect).abs()
+        if epi == 0:
+            assert float((err - expect.abs() * 2.0 ** -8).max()) <= 1e-5
+        else:
+            assert float((err - expect.abs() * 2.0 ** -23).max()) <= 1e-5
+        assert bool((buf[M:] == 7.0).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(64, 1024, 1024), (64, 1024, 2048), (1, 4112, 256),
                                    (37, 1040, 512)])
 @pytest.mark.parametrize("layout", [0, 1])

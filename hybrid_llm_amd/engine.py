@@ -594,7 +594,7 @@ class HybridDecoder:
         else:
             ops.rmsnorm(b["x"], w[p + "ffn_norm"], cfg.eps, out=b["h"])
             from . import _lib
-            s = torch.cuda.current_stream().cuda_stream
+            s = ops._stream()
             _lib.call("llmy_router_topk_bf16", b["h"].data_ptr(),
                       w[p + "router_norm"].data_ptr(), w[p + "w_router"].data_ptr(), None,
                       b["idx"].data_ptr(), b["gates"].data_ptr(), self.B, cfg.d_model,
@@ -700,7 +700,7 @@ class HybridDecoder:
         cfg, w, b = self.cfg, self.w, self.buf
         X, U = b["X"], b["U"]
         ops.mhc_embed(b["tokens"], w["embed"], w["stream_seed"], out=X)
-        s = torch.cuda.current_stream().cuda_stream
+        s = ops._stream()
         kx = cfg.top_k + cfg.shared_experts
         for p, kind, l, st in self._apps():
             self._mhc_read(p, X, "mix_norm", b["raw"], b["maps"], b["h"], b["xb"])
@@ -758,7 +758,7 @@ class HybridDecoder:
         when sampling is configured."""
         from . import _lib
         b, V = self.buf, self.cfg.vocab
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = ops._stream()
         _lib.call("llmy_sample_argmax_f32", b["logits"].data_ptr(), self.B, V,
                   b["next"].data_ptr(), stream)
         if self.sampling is not None:
@@ -887,7 +887,7 @@ class HybridDecoder:
         xb = torch.empty(R, Sm * D, dtype=torch.bfloat16, device=dev)
         raw = torch.empty(R, w["L0.mhc_theta"].shape[0], dtype=torch.float32, device=dev)
         maps = torch.empty(R, Sm + Sm * Sm, dtype=torch.float32, device=dev)
-        s = torch.cuda.current_stream().cuda_stream
+        s = ops._stream()
         E, k = cfg.n_experts, cfg.top_k
         for p, kind, l, st in self._apps():
             self._mhc_read(p, X, "mix_norm", raw, maps, h, xb)
@@ -1014,7 +1014,7 @@ class HybridDecoder:
         cfg, w = self.cfg, self.w
         p = f"L{l}."
         R, D, E, k = x.shape[0], cfg.d_model, cfg.n_experts, cfg.top_k
-        dev, s = self.dev, torch.cuda.current_stream().cuda_stream
+        dev, s = self.dev, ops._stream()
         idx = torch.empty(R, k, dtype=torch.int32, device=dev)
         gates = torch.empty(R, k, dtype=torch.float32, device=dev)
         if self.fused_router_ok:

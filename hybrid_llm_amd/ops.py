@@ -13,7 +13,10 @@ from . import _lib
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current device's current stream as a hipStream_t.  The raw lookup takes 0.2 us;
+    torch.cuda.current_stream() builds a Stream object around it, 2.7 us a call, more
+    than a launch (one token through the MoE layer makes four calls)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:

@@ -172,3 +172,51 @@ def test_top_p_bucket_path_equals_radix_path(kind):
         a = ops().sample_top_p(L, 0.8, p, uc, top_k=0)
         b = ops().sample_top_p(L, 0.8, p, uc, top_k=V)
         assert torch.equal(a, b), (kind, p, torch.nonzero(a != b)[:5])
+
+
+def _deep_rows(kind: str, V: int, g) -> torch.Tensor:
+    """Rows whose mass lies around the 14 octaves that the first histogram covers:
+    log2 distances below the maximum at T = 1."""
+    d = torch.rand(6, V, generator=g) * 46.0            # spread over the whole range
+    if kind == "plateau":                                # most mass beyond 14 octaves
+        d = 14.2 + torch.rand(6, V, generator=g)
+    elif kind == "edge":                                 # on and next to the cut
+        d = 14.0 + (torch.randint(-2, 3, (6, V), generator=g)) * 2.0 ** -18
+    elif kind == "infinite":
+        d[:, ::3] = float("inf")
+    d[:, V // 2] = 0.0
+    d[:, V - 1] = 47.0
+    return -d * 0.6931471805599453
+
+
+@pytest.mark.parametrize("kind", ["spread", "plateau", "edge", "infinite"])
+@pytest.mark.parametrize("V", [32000, 31999, 4100, 37])
+def test_bucket_path_equals_radix_path_deep(kind, V):
+    """The bucket path with ids collected below 14 octaves (and its second pass
+    when a threshold falls there) against the radix path (top_k = V: the same id
+    set) bit for bit, over nuclei and draws that reach every depth."""
+    g = torch.Generator().manual_seed(V)
+    x = _deep_rows(kind, V, g).cuda()
+    for p in (0.3, P90, 0.999, 1.0):
+        for uv in (0.0, 0.05, 0.5, 0.93, 0.999, 0.9999999):
+            u = torch.full((6,), uv).cuda()
+            fast = ops().sample_top_p(x, 1.0, p, u, top_k=0)
+            radix = ops().sample_top_p(x, 1.0, p, u, top_k=V)
+            assert torch.equal(fast, radix), (p, uv, fast, radix)
+
+
+@pytest.mark.parametrize("V", [1, 3, 4, 1023, 16384, 32768, 40001, 70000])
+def test_argmax_first_and_nan(V):
+    """Both load widths and several passes per row: ties, signed zeros, infinities
+    and NaN against numpy (first index of the maximum, the first NaN if any)."""
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(8, V, generator=g).round()
+    x[1] = -float("inf")
+    x[2] = 0.0
+    x[2, V // 2:] = -0.0
+    x[3, V - 1] = float("nan")
+    x[4, V // 3] = float("nan")
+    x[4, V // 2] = float("inf")
+    x[5] = float("nan")
+    x[6, V // 2] = float("inf")
+    assert np.array_equal(ops().argmax(x.cuda()).cpu().numpy(), np.argmax(x.numpy(), axis=1))

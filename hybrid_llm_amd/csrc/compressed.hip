@@ -30,6 +30,8 @@
 //     state is an empty memory and row resets are plain row clears.
 // D layout of a 32x32 MFMA result: lane l, register r holds row
 // (r & 3) + 8 (r >> 2) + 4 (l >> 5), column l & 31.
+#include <algorithm>
+
 #include "common.hpp"
 #include "abi_util.hpp"
 
@@ -205,12 +207,14 @@ __device__ __forceinline__ void topk_regs(const float* srow, int n, int k, int l
   topk_emit(taken, k, lane, sel_s, sel_i, wout, iout);
 }
 
+// kSmall: n <= 1024 (the other paths, and their registers, left out).
+template <bool kSmall = false>
 __device__ __forceinline__ void topk_row(float* srow, int n, int k, int lane, float* wout,
                                          int32_t* iout, float* sel_s, int* sel_i) {
   if (n <= 128) return topk_regs<2>(srow, n, k, lane, wout, iout, sel_s, sel_i);
   if (n <= 256) return topk_regs<4>(srow, n, k, lane, wout, iout, sel_s, sel_i);
   if (n <= 512) return topk_regs<8>(srow, n, k, lane, wout, iout, sel_s, sel_i);
-  if (n <= 1024) return topk_regs<16>(srow, n, k, lane, wout, iout, sel_s, sel_i);
+  if (kSmall || n <= 1024) return topk_regs<16>(srow, n, k, lane, wout, iout, sel_s, sel_i);
   if (n <= 2048) return topk_regs<32>(srow, n, k, lane, wout, iout, sel_s, sel_i);
   float mine = -INFINITY;
   int32_t mine_idx = -1;
@@ -241,6 +245,98 @@ __device__ __forceinline__ void topk_row(float* srow, int n, int k, int lane, fl
 }
 
 // ---------------------------------------------------------------- prefill
+// Top-k selection of 64- and 128-wide heads (NS = Dh / 32) among at most 1024
+// entries: workgroup = (head h, 16-query block, row b), h fastest, 16 waves.  Its
+// score rows take at most 66 KiB and its waves 64 VGPRs each, so two workgroups
+// share a CU at 8 waves per SIMD: one's scores (loads from L2) run beside the
+// other's selections (chains of dependent reductions).  The 32-query kernel below
+// alternates the two phases, the CU waiting half of its cycles: 141 us at 16
+// heads of 128, 4096 tokens, 1024 entries, against 105 here
+// (139 with 8 waves and two rows each).
+// With 2000 entries one 16-query block fills a CU's LDS and the kernel below is
+// the faster one (490 / 505 us at 8000 tokens, 4 heads of 64).
+// Scores are 16 x 16 tiles (v_mfma_f32_16x16x32_bf16: a lane holds 16 bytes of a
+// candidate row, four lanes 64 consecutive ones, four candidates of one query in
+// the result: one 16-byte LDS store), four tiles' rows requested together.
+// Candidates and visibility: the memory rules of the kernel below.
+constexpr int kTopkSmall = 1024;  // most entries of this kernel
+
+template <int NS>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void
+cmp_topk_prefill_kernel(const uint16_t* __restrict__ q, int64_t q_ld,
+                        const uint16_t* __restrict__ k, int64_t k_ld, int T, int n, int H, int W,
+                        int ratio, int top_k, float scale_log2, float* __restrict__ wl,
+                        int32_t* __restrict__ il) {
+  constexpr int Dh = 32 * NS, NW = 16, TP = 2;  // TP tiles' rows are requested together
+  extern __shared__ __align__(16) float sc[];
+  __shared__ float sel_s[NW][kWave];
+  __shared__ int sel_i[NW][kWave];
+  const int h = blockIdx.x % H;
+  const int rest = blockIdx.x / H;
+  const int nqb = (T + 15) / 16;
+  // later query blocks see more entries; they are dispatched first so the
+  // short blocks fill in behind them
+  const int qb = nqb - 1 - rest % nqb;
+  const int b = rest / nqb;
+  const int t0 = qb * 16;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int nc = min(n, min(T, t0 + 16) / ratio);
+  const int ntile = (nc + 15) / 16;
+  // a score row is an odd number of 16-byte units, so the 16 queries of a tile
+  // store to all banks
+  const int ncp = max((nc + 7) & ~7, 8), rsd = ncp + 4;
+  const int t = t0 + r16;
+  const bool q_ok = t < T;
+  const uint16_t* qrow =
+      q + static_cast<int64_t>(b * T + (q_ok ? t : 0)) * q_ld + h * Dh + 8 * g4;
+  const uint16_t* kbase = k + static_cast<int64_t>(b) * n * k_ld + h * Dh + 8 * g4;
+  // entries query t sees: [vlo, vlo + vspan] (an empty interval is out of reach)
+  const int e = (t + 1) / ratio;
+  const int lo = W > 0 ? max(e - W, 0) : 0, hi = min(e, nc) - 1;
+  const bool any = q_ok && lo <= hi;
+  const int vlo = any ? lo : (1 << 30), vspan = any ? hi - lo : 0;
+  uint4 qf[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+    qf[s] = q_ok ? *reinterpret_cast<const uint4*>(qrow + 32 * s) : uint4{0, 0, 0, 0};
+  for (int tile = wave * TP; tile < ntile; tile += NW * TP) {
+    uint4 a[TP][NS];
+#pragma unroll
+    for (int u = 0; u < TP; ++u) {
+      // rows past the candidates re-read the last one (their scores are masked)
+      const uint16_t* kr = kbase + static_cast<int64_t>(min(16 * (tile + u) + r16, nc - 1)) * k_ld;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) a[u][s] = *reinterpret_cast<const uint4*>(kr + 32 * s);
+    }
+    f32x4 acc[TP];
+#pragma unroll
+    for (int u = 0; u < TP; ++u) acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int u = 0; u < TP; ++u)
+        acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[u][s]), as_bf16x8(qf[s]),
+                                                         acc[u], 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < TP; ++u) {
+      const int c0 = 16 * (tile + u) + 4 * g4;
+      f32x4 x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool vis = static_cast<unsigned>(c0 + i - vlo) <= static_cast<unsigned>(vspan);
+        x[i] = vis ? acc[u][i] * scale_log2 : -INFINITY;
+      }
+      if (c0 < ncp) *reinterpret_cast<f32x4*>(sc + r16 * rsd + c0) = x;
+    }
+  }
+  __syncthreads();
+  const int tr = t0 + wave;  // one query row per wave
+  if (tr >= T) return;
+  const int64_t lb = (static_cast<int64_t>(b * T + tr) * H + h) * top_k;
+  topk_row<true>(sc + wave * rsd, nc, top_k, lane, wl + lb, il + lb, sel_s[wave], sel_i[wave]);
+}
+
 // Workgroup = (head h, 32-query block, row b), h fastest; NW waves (top-k: 16,
 // four per SIMD, so the scores' load latency and the selections' scalar
 // chains of one wave hide behind the others' -- the block's score rows fill
@@ -415,6 +511,20 @@ __global__ __launch_bounds__(64 * NW) void cmp_select_prefill_kernel(
     }
     __syncthreads();
   }
+}
+
+// Launch of the 16-query top-k selection (head widths 64 / 128, n <= kTopkSmall).
+void topk_prefill_launch(int B, hipStream_t s, const uint16_t* q, int64_t q_ld, const uint16_t* k,
+                         int64_t k_ld, int T, int n, int H, int Dh, int W, int ratio, int top_k,
+                         float scale_log2, float* wl, int32_t* il) {
+  const dim3 grid(static_cast<unsigned>(B) * ((T + 15) / 16) * H);
+  const size_t lds = static_cast<size_t>(16) * (std::max((n + 7) / 8 * 8, 8) + 4) * sizeof(float);
+  if (Dh == 128)
+    hipLaunchKernelGGL(cmp_topk_prefill_kernel<4>, grid, dim3(1024), lds, s, q, q_ld, k, k_ld, T, n,
+                       H, W, ratio, top_k, scale_log2, wl, il);
+  else
+    hipLaunchKernelGGL(cmp_topk_prefill_kernel<2>, grid, dim3(1024), lds, s, q, q_ld, k, k_ld, T, n,
+                       H, W, ratio, top_k, scale_log2, wl, il);
 }
 
 // Launch of the prefill selection: NS specialised for head widths 64 / 128.
@@ -1372,7 +1482,10 @@ extern "C" int32_t llmy_cmp_memory_prefill_bf16(
   float* wl = static_cast<float*>(workspace);
   int32_t* il = top_k > 0 ? reinterpret_cast<int32_t*>(wl + queries * H * Kmax) : nullptr;
   const size_t lds = static_cast<size_t>(rows) * (ncp + 1) * 4;
-  if (top_k > 0)
+  if (top_k > 0 && (head_dim == 64 || head_dim == 128) && n_entries <= kTopkSmall)
+    topk_prefill_launch(B, s, q, q_ld, mk, mk_ld, T, n_entries, H, head_dim, slots_window, ratio,
+                        top_k, scale * kLog2eC, wl, il);
+  else if (top_k > 0)
     select_prefill_launch<kMemTopK>(dim3(B * nqb * H), lds, s, q, q_ld, mk, mk_ld, T, n_entries,
                                     H, head_dim, slots_window, ratio, top_k, Kmax, rows,
                                     scale * kLog2eC, wl, il);

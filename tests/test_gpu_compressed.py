@@ -103,6 +103,16 @@ def test_memory_prefill(B, T, ratio, H, Dh, Dv, top_k):
     _close(out, _mem_ref(q, kv[:, :Kw], kv[:, Kw:], B, T, ratio, H, Dh, top_k))
 
 
+# The 16-query top-k selection at its edges: one and 15 queries past a block, 1024
+# entries (its most), 1040 (the 32-query kernel), 2200 (there the argmax
+# selection), both head widths.
+@pytest.mark.parametrize("B,T,ratio,H,Dh,top_k", [(2, 17, 1, 2, 128, 8), (1, 31, 2, 3, 64, 16),
+                                                  (1, 1024, 1, 2, 64, 33), (1, 1040, 1, 2, 128, 64),
+                                                  (1, 2200, 1, 1, 64, 16)])
+def test_memory_prefill_topk_blocks(B, T, ratio, H, Dh, top_k):
+    test_memory_prefill(B, T, ratio, H, Dh, 64, top_k)
+
+
 @pytest.mark.parametrize("T,ratio,top_k,levels", [(2048, 4, 32, 3), (2048, 4, 16, 9), (1024, 2, 5, 2)])
 def test_memory_prefill_topk_ties(T, ratio, top_k, levels):
     """Scores drawn from a few levels, so many summaries tie at the top-k

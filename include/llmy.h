@@ -179,8 +179,8 @@ int32_t llmy_banded_attn_decode_parts_bf16(const float* parts, int32_t nparts,
 /* --- Gated delta rule, prefill (chunked; model/layers/gated_deltanet.py:140-149) */
 
 /* Workspace (bytes) that llmy_gdn_prefill_bf16 needs for (B, T, H, dk, dv):
- * per 64-token chunk W [64,dk], U0 [64,dv], A [64,64] and 2 x 64 decay
- * factors, fp32.  No counterpart in the reference. */
+ * per 64-token chunk 64 (dk + dv + 66) fp32 words, an upper bound of the chunk's
+ * inverse and per-token factors.  No counterpart in the reference. */
 int64_t llmy_gdn_prefill_workspace_bytes(int32_t B, int32_t T, int32_t H, int32_t dk,
                                          int32_t dv);
 

@@ -334,6 +334,8 @@ struct FastLds {
   int32_t id;
 };
 
+// x: a logit of the row (x <= r.m, or NaN) or -infinity, so the bucket is one of
+// 0 .. kFastBins - 1.
 __device__ __forceinline__ int fast_bin(float x, NucRow r) {
   if (x == r.m) return 0;
   const float d = ((r.m - x) * r.c) * r.b;
@@ -441,7 +443,8 @@ __device__ __forceinline__ bool fast_top_p(const float* x, uint32_t live, NucRow
 #pragma unroll
   for (int j = 0; j < kNucPer; ++j) {
     const float xj = nuc_x(x, j);
-    const u64 w = nuc_weight<false>(xj, live, j, r);  // 0 for ids outside the row
+    const u64 w = nuc_weight<false>(xj, live, j, r);
+    if (w == 0ull) continue;  // ids outside the row among them: no atomics for nothing
     const int bin = fast_bin(xj, r);
     if (bin < cut)
       atomicAdd(&fs.mass[bin], w);
@@ -502,7 +505,8 @@ __device__ __forceinline__ bool fast_top_p(const float* x, uint32_t live, NucRow
   return true;
 }
 
-// The thread's 32 logits.  kSpread: element 4 q + i is id 4 (t + 1024 q) + i
+// The thread's 32 logits, -infinity for ids outside the row (the row's maximum
+// may lie below any other filler: fast_bin needs x <= max).  kSpread: element 4 q + i is id 4 (t + 1024 q) + i
 // (without kVec4: element j is id t + 1024 j), so a wave's load covers whole
 // lines; else ids 32 t .. 32 t + 31, the order the radix path's tie scan needs
 // (each lane 128 bytes apart: a wave's load touches 64 lines, and the 16 waves'
@@ -521,7 +525,7 @@ __device__ __forceinline__ uint32_t nuc_load(const float* row, int V, float* x) 
 #pragma unroll
     for (int q = 0; q < kNucPer / 4; ++q) {
       const int i = nuc_id<kVec4, kSpread>(4 * q);
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+      float4 v = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
       if (i < V) v = *reinterpret_cast<const float4*>(row + i);  // V % 4 == 0
       x[4 * q] = v.x;
       x[4 * q + 1] = v.y;
@@ -532,7 +536,7 @@ __device__ __forceinline__ uint32_t nuc_load(const float* row, int V, float* x) 
 #pragma unroll
     for (int j = 0; j < kNucPer; ++j) {
       const int i = nuc_id<kVec4, kSpread>(j);
-      x[j] = i < V ? row[i] : 0.f;
+      x[j] = i < V ? row[i] : -INFINITY;
     }
   }
 #pragma unroll

@@ -205,6 +205,26 @@ def test_bucket_path_equals_radix_path_deep(kind, V):
             assert torch.equal(fast, radix), (p, uv, fast, radix)
 
 
+@pytest.mark.parametrize("spread", [0.01, 3.0, 30.0])
+@pytest.mark.parametrize("shift", [-2.0, -1000.0])
+@pytest.mark.parametrize("V", [1, 37, 4100, 31999])
+def test_top_p_rows_below_zero(V, shift, spread):
+    """Rows whose maximum lies below zero (log-probabilities) and that leave threads
+    without ids: the ids past the row must reach no bucket.  Against the radix path
+    bit for bit, and against the oracle."""
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(16, V, generator=g) * spread
+    x = x - x.max(-1, keepdim=True).values + shift
+    u = torch.rand(16, generator=g)
+    for p in (0.3, P90, 1.0):
+        fast = ops().sample_top_p(x.cuda(), 0.8, p, u.cuda(), top_k=0)
+        radix = ops().sample_top_p(x.cuda(), 0.8, p, u.cuda(), top_k=V)
+        assert torch.equal(fast, radix), (p, fast, radix)
+    # 0.01 apart, some 1e4 ids share the mass and 2^-14 steps of the logits: fewer
+    # rows' draws are decided beyond the bound
+    _check(x, 0.8, P90, u, 0, min_exact=0.0 if spread < 1 else 0.6)
+
+
 @pytest.mark.parametrize("V", [1, 3, 4, 1023, 16384, 32768, 40001, 70000])
 def test_argmax_first_and_nan(V):
     """Both load widths and several passes per row: ties, signed zeros, infinities

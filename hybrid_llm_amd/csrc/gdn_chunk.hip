@@ -284,17 +284,27 @@ __device__ __forceinline__ int v_swz(int t) {
 }
 
 // One copy into LDS: 16 (or 4) bytes per lane from rsrc + off to dst + lane *
-// 16 (4).  Lanes past the buffer's range read zero.  In inline asm so that
+// 16 (4).  What lanes past the buffer's range leave in LDS is not relied on
+// (the kernel clears the rows of a ragged chunk first).  In inline asm so that
 // the compiler does not make every later LDS read of the wave wait for it; the
-// wave waits (vmcnt) before the barrier that publishes the data.
+// wave waits (vmcnt) before the barrier that publishes the data.  The compiler
+// inserts no wait states for what is inside: s_nop 3 after the move of m0 makes
+// the five that a buffer load needs after a VALU write of its descriptor (a
+// readfirstlane, or a v_readlane that restores a spilled SGPR).  m0 is reserved
+// (nothing is allocated to it, hence the compiler's warning), but the compiler
+// itself keeps values there for LDS-DMA builtins and indexed moves: the clobber
+// tells it that they are gone.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void lds_copy16(const u32x4& rsrc, uint32_t off, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               ::"s"(dst), "v"(off), "s"(rsrc) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               ::"s"(dst), "v"(off), "s"(rsrc) : "memory", "m0");
 }
 __device__ __forceinline__ void lds_copy4(const u32x4& rsrc, uint32_t off, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-               ::"s"(dst), "v"(off), "s"(rsrc) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, 0 offen lds"
+               ::"s"(dst), "v"(off), "s"(rsrc) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 __device__ __forceinline__ u32x4 buffer_of(const void* p, uint32_t bytes) {
   const uint64_t a = reinterpret_cast<uint64_t>(p);

@@ -138,6 +138,16 @@ __device__ __forceinline__ uint32_t order_key(float f) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
+// Order this wave's LDS accesses before against those after, for data that its
+// lanes pass to each other: a wave's LDS operations complete in order, so only the
+// compiler has to keep them so (it sees no dependence between different lanes'
+// addresses).  No instruction is emitted.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // (value, index) packed so that an unsigned max picks the largest value and,
 // among equal values, the lowest index.
 __device__ __forceinline__ uint64_t value_index_key(float f, uint32_t idx) {

@@ -119,6 +119,7 @@ __device__ __forceinline__ void tile_store(const TileArgs& a, const f32x16 (&acc
         else
           *reinterpret_cast<float4*>(w) = make_float4(v0, v1, v2, v3);
       }
+    wave_lds_order();  // the block is written: other lanes' values are read below
     const int mb = m0 + row_of(i);
 #pragma unroll
     for (int t0 = 0; t0 < IT; t0 += 4) {
@@ -162,6 +163,7 @@ __device__ __forceinline__ void tile_store(const TileArgs& a, const f32x16 (&acc
                                                       r.z + v.z * g.z, r.w + v.w * g.w);
       }
     }
+    wave_lds_order();  // the block is read: the next one takes its place
   }
 }
 

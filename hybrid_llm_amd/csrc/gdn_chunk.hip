@@ -159,10 +159,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_prep_kernel(
     f[4 * kC] = sc;
     f[5 * kC] = static_cast<float>(sg);
   }
-  // one wave: its LDS operations complete in order, only the compiler must
-  // keep them so
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_order();
 
   // ---- N = I + L: block (m, j) in D form (rows 4 g4 + i of m, column r16 of j)
   f32x4 nb[4][4];
@@ -188,8 +185,7 @@ __global__ __launch_bounds__(64) void gdn_chunk_prep_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) dg[m * BD + (4 * g4 + i) * PD + r16] = nb[m][m][i];
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_order();
 
   // ---- the diagonal blocks' inverses: lane (block g4, column r16)
   {
@@ -207,12 +203,11 @@ __global__ __launch_bounds__(64) void gdn_chunk_prep_kernel(
       }
       x[t] = t < r16 ? 0.f : (a[0] + a[1]) + (a[2] + a[3]);
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_order();
 #pragma unroll
     for (int t = 0; t < 16; ++t) dg[g4 * BD + t * PD + r16] = x[t];
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_order();
 
   // ---- T_ij^T in D form; row block i needs only N and its own T_im, m > j
   f32x4 tt[4][4], tj[3];

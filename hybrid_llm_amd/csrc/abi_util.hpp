@@ -24,6 +24,19 @@ inline bool aligned(const void* p, size_t a) {
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
+// Compute units of the device that was current at the first call (256 where it
+// does not say), asked for once per process; any thread may be the first.
+inline int compute_units() {
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    const bool ok = hipGetDevice(&dev) == hipSuccess &&
+                    hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) ==
+                        hipSuccess && n > 0;
+    return ok ? n : 256;
+  }();
+  return cus;
+}
+
 inline int32_t launch_status() { return static_cast<int32_t>(hipGetLastError()); }
 
 }  // namespace llmy

@@ -381,25 +381,13 @@ struct TileShape {
 constexpr TileShape kTileShapes[] = {
     {128, 128, 1.f}, {128, 192, 1.43f}, {128, 256, 1.68f}, {256, 192, 2.46f}, {256, 256, 2.93f}};
 
-// Compute units of the current device (queried once per process).
-int dense_cus() {
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    return n;
-  }();
-  return cus;
-}
-
 // Modelled time of out[M, N] with a shape: whole rounds of workgroups (a second
 // 128 x 128 tile per CU shares the CU with the first: 384 tiles took 18.6 us, 480
 // 21.4, 768 33.9 against 11.7 for 256).
 float tile_cost(int shape, int M, int N) {
   const TileShape& t = kTileShapes[shape];
   const long long tiles = static_cast<long long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-  const float rounds = static_cast<float>((tiles + dense_cus() - 1) / dense_cus());
+  const float rounds = static_cast<float>((tiles + compute_units() - 1) / compute_units());
   return shape == 0 ? 0.15f + 0.85f * rounds : t.round * rounds;
 }
 

@@ -713,21 +713,6 @@ extern "C" int64_t llmy_gdn_prefill_workspace_bytes(int32_t B, int32_t T, int32_
 
 namespace {
 
-// The prep + scan launches over a caller-sized workspace (validated by the
-// entry points below).
-// Compute units of the current device (queried once per process).
-int device_cus() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cus = n;
-  }
-  return cus;
-}
-
 template <int D, int NW>
 void launch_scan(const llmy_bf16* q, const llmy_bf16* k, const llmy_bf16* v, const uint16_t* Tf,
                  const float* fac, float* state, llmy_bf16* out, int B, int T, int H, int NC,
@@ -738,6 +723,8 @@ void launch_scan(const llmy_bf16* q, const llmy_bf16* k, const llmy_bf16* v, con
                      aligned(out, 8) ? 1 : 0);
 }
 
+// The prep + scan launches over a caller-sized workspace (validated by the
+// entry points below).
 template <int D>
 int32_t gdn_prefill_run(const llmy_bf16* q, const llmy_bf16* k, const llmy_bf16* v,
                         const float* beta, const float* g, const int32_t* reset, float* state,
@@ -757,7 +744,7 @@ int32_t gdn_prefill_run(const llmy_bf16* q, const llmy_bf16* k, const llmy_bf16*
   // of 128, us for NW = 1 / 2 / 4: 1 x 4096 tokens, 128 column tiles: 141 / 155
   // / 208; 4 x 1024, 512 tiles: 83 / 54 / 64; 8 x 2048, 1024 tiles: 289 / 175 /
   // 133).
-  const long long cols = static_cast<long long>(B) * H * (D / 16), cus = device_cus();
+  const long long cols = static_cast<long long>(B) * H * (D / 16), cus = compute_units();
   if (cols <= cus)
     launch_scan<D, 1>(q, k, v, Tf, fac, state, out, B, T, H, NC, s);
   else if (cols <= 2 * cus)

@@ -510,17 +510,7 @@ static int32_t launch_grouped(const GroupedArgs& g, int grid, hipStream_t s) {
 }
 
 // One persistent workgroup per CU (a multiple of 8: an equal share per XCD).
-static int grouped_grid() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cus = n;
-  }
-  return std::max(kGXcd, cus / kGXcd * kGXcd);
-}
+static int grouped_grid() { return std::max(kGXcd, compute_units() / kGXcd * kGXcd); }
 
 // Both grouped GEMMs of one MoE prefill (gate_up + SwiGLU into act, then the
 // gate-scaled down projection into y).  Validated by the caller: D % 256 == 0,

@@ -1,8 +1,9 @@
-"""Inline assembly of the kernels, read as source: what the compiler does not check.
+"""The kernels' and entry points' source: what the compiler does not check.
 
 The compiler treats an asm statement as one opaque instruction.  A register it writes
 must be named as clobbered, and the wait states that the hardware asks for between its
-operands' writers and its own memory instruction must be inside it.
+operands' writers and its own memory instruction must be inside it.  An entry point may be called by any thread, so a value that a
+function keeps is initialised where it is declared.
 """
 import re
 from pathlib import Path
@@ -46,3 +47,12 @@ def test_buffer_loads_wait_for_their_descriptor():
             nop = re.match(r"s_nop\s+(\d+)", ins)
             waits += int(nop.group(1)) + 1 if nop else 1
     assert seen >= 2
+
+
+def test_function_statics_are_initialised_once():
+    """A function-local ``static`` scalar that is filled in later is read and written by
+    every thread that calls; const ones are initialised under the language's guard."""
+    for path in sorted(CSRC.glob("*.hip")) + sorted(CSRC.glob("*.hpp")) + sorted(CSRC.glob("*.cpp")):
+        for line in path.read_text().splitlines():
+            assert not re.match(r"\s+static\s+(int|bool|long long|unsigned|void\s*\*)\s+\w+\s*=", line), (
+                path.name, line)

@@ -16,6 +16,7 @@
 // contiguous range of them, so the tiles an XCD runs together share few x
 // and weight tiles in its L2.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "abi_util.hpp"
@@ -216,7 +217,17 @@ __device__ __forceinline__ void settle_frags(u32x4 (&f)[N]) {
 // vmcnt <= n, expcnt and lgkmcnt left open.
 constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
 
-template <int BM, int BN, int NS, int OCC, int EPI>
+// BLK: the sums restart every 256 k (kSumSteps) and the block sums are added in
+// order, the sums of the weight-streaming kernel: bit for bit at K <= 2048, where
+// it has a wave per 256 k, so a row's outputs do not change where this kernel takes
+// over.  One chain over all of K is 2 to 3 times further from 64 bits (relative
+// error at K = 512 / 1024 / 2048 / 4096, fp32 out: 1.25e-7 / 1.84e-7 / 2.71e-7 /
+// 3.95e-7 in one chain, 0.90e-7 / 0.95e-7 / 1.03e-7 / 1.15e-7 in blocks), and the
+// blocks cost nothing: 96 x 1024 x 1024 takes 8.8 us, in one chain 9.6 (only where
+// the chip is full do they: 255 x 32000 x 1024 22.1, 21.1).
+constexpr int kSumSteps = 8;
+
+template <int BM, int BN, int NS, int OCC, int EPI, bool BLK>
 __global__ __launch_bounds__(kThreads, OCC) void tile_gemm_kernel(TileArgs a) {
   constexpr int FA = BM / 64, FB = BN / 64, NF = FA + FB, NM = FA * FB;
   constexpr int A_STAGE = BM * 64, STAGE = (BM + BN) * 64;
@@ -286,13 +297,16 @@ __global__ __launch_bounds__(kThreads, OCC) void tile_gemm_kernel(TileArgs a) {
   } while (0)
 #define TILE_FENCE() __builtin_amdgcn_sched_barrier(0)
 
-  f32x16 acc[FA][FB];
+  f32x16 acc[FA][FB], sum[FA][FB];  // sum: BLK only
 #pragma unroll
   for (int i = 0; i < FA; ++i)
 #pragma unroll
     for (int j = 0; j < FB; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      for (int r = 0; r < 16; ++r) {
+        acc[i][j][r] = 0.f;
+        if constexpr (BLK) sum[i][j][r] = 0.f;
+      }
 
   // steps 0 .. NS - 2 and step NS - 1's x copies in flight
 #pragma unroll
@@ -314,14 +328,17 @@ __global__ __launch_bounds__(kThreads, OCC) void tile_gemm_kernel(TileArgs a) {
 #pragma unroll
   for (int n = 0; n < NF; ++n) TILE_READ(h0, n, 0u, 0);
   settle_frags(h0);
-  for (int kk = 0; kk < nk; ++kk) {
+  // one step; FIRST and LAST: of a block of k (BLK), whose products start from zero
+  // and join the sums behind the last step's MFMAs
+  auto step = [&](int kk, auto FIRST, auto LAST) {
     const int kb = min(kk + NS - 1, nk - 1), ka = min(kk + NS, nk - 1);
     const char* const bb = b_base + static_cast<long long>(b_step) * kb;
     const char* const ab = a_base + 64 * ka;
 #pragma unroll
     for (int n = 0; n < NM; ++n) {
+      f32x16& c = acc[n / FB][n % FB];
       TILE_FENCE();
-      acc[n / FB][n % FB] = mfma32(h0[FA + n % FB], h0[n / FB], acc[n / FB][n % FB]);
+      c = mfma32(h0[FA + n % FB], h0[n / FB], FIRST.value ? f32x16{0.f} : c);
       TILE_FENCE();
       if (n < NF) TILE_READ(h1, n, off, 1);
       if (n % 2 == 1 && n / 2 < LB) dma16(bb + bo[n / 2], b_dst + last + 1024 * (n / 2));
@@ -342,11 +359,26 @@ __global__ __launch_bounds__(kThreads, OCC) void tile_gemm_kernel(TileArgs a) {
       TILE_FENCE();
       if (n < NF) TILE_READ(h0, n, off, 0);
       if (n % 2 == 1 && n / 2 < LA) dma16(ab + ao[n / 2], a_dst + last + 1024 * (n / 2));
+      if constexpr (LAST.value) {
+        if (n > 0) sum[(n - 1) / FB][(n - 1) % FB] += acc[(n - 1) / FB][(n - 1) % FB];
+      }
     }
     TILE_FENCE();
+    if constexpr (LAST.value) sum[FA - 1][FB - 1] += acc[FA - 1][FB - 1];
     // no read of the loop is in flight across its edge: the compiler knows
     // nothing of them and may move a register that one is still to fill
     settle_frags(h0);
+  };
+  constexpr std::true_type yes;
+  constexpr std::false_type no;
+  if constexpr (BLK) {
+    for (int kk = 0; kk < nk; kk += kSumSteps) {  // K % 256 == 0: whole blocks
+      step(kk, yes, no);
+      for (int i = 1; i < kSumSteps - 1; ++i) step(kk + i, no, no);
+      step(kk + kSumSteps - 1, no, yes);
+    }
+  } else {
+    for (int kk = 0; kk < nk; ++kk) step(kk, no, no);
   }
 #undef TILE_FENCE
 #undef TILE_READ
@@ -356,14 +388,15 @@ __global__ __launch_bounds__(kThreads, OCC) void tile_gemm_kernel(TileArgs a) {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   static_assert(4 * 32 * (FB * 128 + 16) <= NS * STAGE, "epilogue rows");
-  tile_store<EPI, FA, FB>(a, acc, m0, n0, [&](int i) { return 32 * (FA * wm + i); }, 32 * FB * wn,
-                          lane, smem + wave * 32 * (FB * 128 + 16));
+  tile_store<EPI, FA, FB>(a, BLK ? sum : acc, m0, n0, [&](int i) { return 32 * (FA * wm + i); },
+                          32 * FB * wn, lane, smem + wave * 32 * (FB * 128 + 16));
 }
 
-template <int BM, int BN, int NS, int OCC, int EPI>
+template <int BM, int BN, int NS, int OCC, int EPI, bool BLK>
 int32_t launch_tiles(const TileArgs& g, long long items, hipStream_t s) {
   const unsigned grid = static_cast<unsigned>((items + kNumXcd - 1) / kNumXcd * kNumXcd);
-  hipLaunchKernelGGL((tile_gemm_kernel<BM, BN, NS, OCC, EPI>), dim3(grid), dim3(kThreads), 0, s, g);
+  hipLaunchKernelGGL((tile_gemm_kernel<BM, BN, NS, OCC, EPI, BLK>), dim3(grid), dim3(kThreads), 0, s,
+                     g);
   return launch_status();
 }
 
@@ -391,11 +424,15 @@ float tile_cost(int shape, int M, int N) {
   return shape == 0 ? 0.15f + 0.85f * rounds : t.round * rounds;
 }
 
-// The cheapest shape.  Every shape sums each output over k in the same order,
-// so the results do not depend on the choice.
+// Rows below which outputs are summed in 256-wide blocks of k (tiles of 128 rows
+// only: the second set of sums takes registers that the larger ones do not have).
+constexpr int kBlockSumRows = 256;
+
+// The cheapest shape.  Every shape that a row count allows sums each output over k
+// in the same order, so the results do not depend on the choice.
 int tile_shape(int M, int N) {
   int best = 0;
-  for (int i = 1; i < 5; ++i)
+  for (int i = 1; i < (M < kBlockSumRows ? 3 : 5); ++i)
     if (tile_cost(i, M, N) < tile_cost(best, M, N)) best = i;
   return best;
 }
@@ -438,19 +475,27 @@ int32_t dense_gemm_mfma(const uint16_t* x, const uint16_t* w, void* out, const f
   const long long items = static_cast<long long>(g.m_tiles) * g.n_tiles;
   if (items >= (1ll << 31) - kNumXcd) return static_cast<int32_t>(hipErrorInvalidValue);
   int32_t st = 0;
-#define LLMY_DENSE(BM_, BN_, NS_, OCC_)                                                    \
-  switch (epi) {                                                                           \
-    case kDenseBf16: st = launch_tiles<BM_, BN_, NS_, OCC_, kDenseBf16>(g, items, s); break; \
-    case kDenseF32: st = launch_tiles<BM_, BN_, NS_, OCC_, kDenseF32>(g, items, s); break;   \
-    case kDenseResid: st = launch_tiles<BM_, BN_, NS_, OCC_, kDenseResid>(g, items, s); break; \
-    default: st = launch_tiles<BM_, BN_, NS_, OCC_, kDenseGated>(g, items, s); break;      \
+#define LLMY_DENSE(BM_, BN_, NS_, OCC_, BLK_)                                                  \
+  switch (epi) {                                                                              \
+    case kDenseBf16: st = launch_tiles<BM_, BN_, NS_, OCC_, kDenseBf16, BLK_>(g, items, s); break;   \
+    case kDenseF32: st = launch_tiles<BM_, BN_, NS_, OCC_, kDenseF32, BLK_>(g, items, s); break;     \
+    case kDenseResid: st = launch_tiles<BM_, BN_, NS_, OCC_, kDenseResid, BLK_>(g, items, s); break; \
+    default: st = launch_tiles<BM_, BN_, NS_, OCC_, kDenseGated, BLK_>(g, items, s); break;          \
   }
-  switch (shape) {
-    case 0: LLMY_DENSE(128, 128, 5, 2) break;
-    case 1: LLMY_DENSE(128, 192, 7, 1) break;
-    case 2: LLMY_DENSE(128, 256, 6, 1) break;
-    case 3: LLMY_DENSE(256, 192, 5, 1) break;
-    default: LLMY_DENSE(256, 256, 5, 1) break;
+  if (M < kBlockSumRows) {
+    switch (shape) {
+      case 0: LLMY_DENSE(128, 128, 5, 2, true) break;
+      case 1: LLMY_DENSE(128, 192, 7, 1, true) break;
+      default: LLMY_DENSE(128, 256, 6, 1, true) break;
+    }
+  } else {
+    switch (shape) {
+      case 0: LLMY_DENSE(128, 128, 5, 2, false) break;
+      case 1: LLMY_DENSE(128, 192, 7, 1, false) break;
+      case 2: LLMY_DENSE(128, 256, 6, 1, false) break;
+      case 3: LLMY_DENSE(256, 192, 5, 1, false) break;
+      default: LLMY_DENSE(256, 256, 5, 1, false) break;
+    }
   }
 #undef LLMY_DENSE
   if (st != 0 || g.N == N) return st;

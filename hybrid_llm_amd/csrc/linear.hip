@@ -623,10 +623,12 @@ int32_t dense_gemm_mfma(const uint16_t* x, const uint16_t* w, void* out, const f
 
 // Rows from which the dense projections switch from the weight-streaming
 // kernel (every weight byte read once per 64 rows, HBM-bound) to the MFMA
-// tiles (compute-bound); decode batches stay below it.  us, bf16 out, packed
-// weights, streaming / tiles: 65 x 3072 x 1024 10.1 / 9.7, 65 x 1024 x 2048 15.1 /
-// 16.2, 96 x 1024 x 2048 17.4 / 16.4, 128 x 4112 x 1024 19.2 / 10.1, 255 x 1024 x
-// 1024 21.1 / 9.7, gated residual 30.2 / 13.0.
+// tiles (compute-bound).  Up to 255 rows the tiles sum in the streaming
+// kernel's order, so the switch changes no bits up to K = 2048.  The line lies at
+// the fewest rows where no width loses: us, bf16 out, packed weights, streaming /
+// tiles at 96 rows: N x K = 16 x 256 6.1 / 4.2, 256 x 1024 10.5 / 8.7, 1024 x 2048
+// 16.4 / 14.7, 256 x 4096 29.5 / 26.3, 4112 x 1024 16.1 / 9.1; gated residual 256 x
+// 256 9.3 / 7.7; 255 rows, 1024 x 1024 21.1 / 8.9, gated residual 30.2 / 12.4.
 constexpr int kDenseMfmaMinRows = 96;
 
 }  // namespace llmy

@@ -106,6 +106,32 @@ def test_linear_tile_shapes(M, N, K, epi):
         assert bool((buf[M:] == 7.0).all())
 
 
+# The tiles take over from the streaming kernel at 96 rows; below 256 rows (and up to
+# K = 2048) they sum in its order, so a row has the same bits in any batch.
+@pytest.mark.parametrize("M", [96, 130, 255])
+@pytest.mark.parametrize("N,K", [(16, 256), (768, 256), (1040, 512), (1024, 768), (3072, 1024),
+                                 (4112, 1024), (1024, 2048), (24400, 512), (32000, 256)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+def test_linear_rows_do_not_depend_on_the_batch(M, N, K, epi):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = _bf(torch.randn(M, K, generator=g, device="cuda"))
+    w = _bf(torch.randn(N, K, generator=g, device="cuda") * 0.02)
+    base = torch.randn(M, N, generator=g, device="cuda")
+    aux = torch.rand(M, N, generator=g, device="cuda")
+    for layout in (0, 1):
+        if layout == 1 and N >= 8192:
+            continue  # up to 64 rows of packed weights run another kernel there
+        wl = w if layout == 0 else ops().pack_weights(w)
+
+        def rows(lo, hi):
+            out = base[lo:hi].clone() if epi >= 2 else None
+            return ops().linear(x[lo:hi].clone(), wl, out=out, epilogue=epi,
+                                aux=aux[lo:hi].clone() if epi == 3 else None, layout=layout)
+
+        parts = torch.cat([rows(lo, min(M, lo + 64)) for lo in range(0, M, 64)])
+        assert torch.equal(rows(0, M), parts)
+
+
 @pytest.mark.parametrize("M,N,K", [(64, 1024, 1024), (64, 1024, 2048), (1, 4112, 256),
                                    (37, 1040, 512)])
 @pytest.mark.parametrize("layout", [0, 1])

@@ -172,9 +172,11 @@ __device__ __forceinline__ void tile_store(const TileArgs& a, const f32x16 (&acc
 // 32 k per step through a ring of NS stages.  A stage holds the BM rows of x
 // (64 bytes each, 16-byte chunks XOR-swizzled by row: the 16 lanes that a
 // ds_read_b128 serves at once take 16 rows at one chunk index and meet all bank
-// groups) and BN / 16 weight fragments of 16 rows x 32 k (1 KiB, lane l: row l %
-// 16 at k 8 (l / 16) .. +7, the packed operand order), all by
-// global_load_lds_dwordx4 from scalar bases plus 32-bit lane offsets; every
+// groups) and the BN weight rows: packed ones as BN / 16 fragments of 16 rows x 32 k
+// (1 KiB, lane l: row l % 16 at k 8 (l / 16) .. +7), row-major ones like those of x
+// (in fragments an instruction would gather 64 pieces of 16 bytes, four rows' worth
+// of lanes apart: 96 x 1024 x 4096 39.9 -> 28.7 us, 4096 x 1024 x 1024 15.2 -> 13.0).
+// All by global_load_lds_dwordx4 from scalar bases plus 32-bit lane offsets; every
 // wave issues the same copies each step (past the last step they re-read it),
 // so its waits count fixed numbers.
 //
@@ -264,9 +266,12 @@ __global__ __launch_bounds__(kThreads, OCC) void tile_gemm_kernel(TileArgs a) {
   }
 #pragma unroll
   for (int q = 0; q < LB; ++q) {
-    const int n = min(n0 + 16 * (LB * wave + q) + (lane & 15), a.N - 1);
-    bo[q] = static_cast<uint32_t>((packed ? packed_at(n, 8 * (lane >> 4), K)
-                                          : static_cast<long long>(n) * K + 8 * (lane >> 4)) * 2);
+    const int nb = n0 + 16 * (LB * wave + q);
+    const long long at =
+        packed ? packed_at(min(nb + (lane & 15), a.N - 1), 8 * (lane >> 4), K)
+               : static_cast<long long>(min(nb + (lane >> 2), a.N - 1)) * K +
+                     8 * ((lane & 3) ^ (lane >> 4));
+    bo[q] = static_cast<uint32_t>(at * 2);
   }
   const char* const a_base = reinterpret_cast<const char*>(a.x);
   const char* const b_base = reinterpret_cast<const char*>(a.w);
@@ -277,22 +282,25 @@ __global__ __launch_bounds__(kThreads, OCC) void tile_gemm_kernel(TileArgs a) {
   const uint32_t base = lds_addr(smem);
   const uint32_t xa0 = base + wm * (BM * 32) + lr * 64 + ((lh ^ ((lr >> 2) & 3)) << 4);
   const uint32_t xa1 = base + wm * (BM * 32) + lr * 64 + (((2 + lh) ^ ((lr >> 2) & 3)) << 4);
-  const uint32_t xb = base + A_STAGE + (2 * FB * wn + (lr >> 4)) * 1024 + lh * 256 + (lane & 15) * 16;
+  const uint32_t xb = base + A_STAGE + wn * (BN * 32);
+  const uint32_t xb0 = xb + (packed ? (lr >> 4) * 1024 + lh * 256 + (lane & 15) * 16
+                                    : lr * 64 + ((lh ^ ((lr >> 2) & 3)) << 4));
+  const uint32_t xb1 = packed ? xb0 + 512 : xb + lr * 64 + (((2 + lh) ^ ((lr >> 2) & 3)) << 4);
   // fragment n of k half H of the stage at byte offset o: n < FA: rows BM / 2 wm
   // + 32 n of x, else the wave's 32-column weight block n - FA
 #define TILE_READ(F, n, o, H)                                           \
   do {                                                                 \
-    const uint32_t a_ = ((H) ? xa1 : xa0) + (o), b_ = xb + (o);        \
+    const uint32_t a_ = ((H) ? xa1 : xa0) + (o), b_ = ((H) ? xb1 : xb0) + (o); \
     if ((n) < FA) {                                                    \
       if ((n) == 0) F[0] = lds_frag<0>(a_);                            \
       if ((n) == 1) F[1] = lds_frag<2048>(a_);                         \
       if ((n) == 2) F[2] = lds_frag<4096>(a_);                         \
       if ((n) == 3) F[3] = lds_frag<6144>(a_);                         \
     } else {                                                           \
-      if ((n) == FA) F[FA] = lds_frag<512 * (H)>(b_);                  \
-      if ((n) == FA + 1) F[FA + 1] = lds_frag<2048 + 512 * (H)>(b_);   \
-      if ((n) == FA + 2) F[NF > FA + 2 ? FA + 2 : 0] = lds_frag<4096 + 512 * (H)>(b_); \
-      if ((n) == FA + 3) F[NF > FA + 3 ? FA + 3 : 0] = lds_frag<6144 + 512 * (H)>(b_); \
+      if ((n) == FA) F[FA] = lds_frag<0>(b_);                          \
+      if ((n) == FA + 1) F[FA + 1] = lds_frag<2048>(b_);               \
+      if ((n) == FA + 2) F[NF > FA + 2 ? FA + 2 : 0] = lds_frag<4096>(b_); \
+      if ((n) == FA + 3) F[NF > FA + 3 ? FA + 3 : 0] = lds_frag<6144>(b_); \
     }                                                                  \
   } while (0)
 #define TILE_FENCE() __builtin_amdgcn_sched_barrier(0)

@@ -13,53 +13,60 @@
 
 namespace llmy {
 
-// One 1024-thread workgroup per row, latency-bound: a thread's 32 ids of a pass
-// are requested together (float4 where rows allow it), it keeps the first of its
+// One 1024-thread workgroup per row, latency-bound: a thread's 32 (16) ids of a
+// pass are requested together (float4 where rows allow it), it keeps the first of its
 // largest values by plain compares (a NaN wins and stays), and only that one
-// becomes a packed (value, index) key for the wave and block reductions.
-// 64 x 32000, calls back to back: 8.6 -> 5.7 us (a key per element and 4-byte
-// loads before).
+// becomes a packed (value, index) key for the wave and block reductions.  A pass
+// runs in groups of 4096 ids and skips those that start past the row.  Calls back to
+// back on three sets of logits in turn, us, a key per element and 4-byte loads ->
+// this: 64 x 32000 6.3 -> 5.1, 64 x 31999 6.3 -> 5.6, 64 x 128256 19.0 -> 13.3, 64 x
+// 16384 4.1 -> 3.7; from 8192 ids down both take a launch's 3.5 (4.6 with passes that
+// always covered 32768 ids).
 template <bool kVec4>
 __global__ __launch_bounds__(1024) void argmax_rows_kernel(const float* __restrict__ logits,
-                                                           int V, int32_t* __restrict__ out) {
+                                                           int rowlen, int32_t* __restrict__ out) {
   __shared__ uint64_t part[16];
-  constexpr int kPer = kVec4 ? 32 : 16;
-  const float* row = logits + static_cast<size_t>(blockIdx.x) * V;
-  const int t = threadIdx.x;
+  constexpr uint32_t kGroups = kVec4 ? 8 : 4, kGroup = 4 * 1024;
+  const float* row = logits + static_cast<size_t>(blockIdx.x) * rowlen;
+  const uint32_t V = rowlen, t = threadIdx.x;  // unsigned: the last pass may end past 2^31
   float best = -INFINITY;
-  int at = -1;
-  for (int base = 0; base < V; base += kPer * 1024) {
-    float v[kPer];
-    if (kVec4) {
+  uint32_t at = 0;
+  bool any = false;
+  for (uint32_t base = 0; base < V; base += kGroups * kGroup) {
+    float v[kGroups][4];
 #pragma unroll
-      for (int q = 0; q < kPer / 4; ++q) {
-        const int i = base + 4 * (t + 1024 * q);
-        const float4 w = i < V ? *reinterpret_cast<const float4*>(row + i)  // V % 4 == 0
-                               : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-        v[4 * q] = w.x;
-        v[4 * q + 1] = w.y;
-        v[4 * q + 2] = w.z;
-        v[4 * q + 3] = w.w;
-      }
-    } else {
+    for (uint32_t q = 0; q < kGroups; ++q) {
+      if (base + q * kGroup >= V) continue;  // uniform
+      const uint32_t i0 = base + q * kGroup + (kVec4 ? 4 * t : t);
+      if (kVec4) {
+        const float4 w = i0 < V ? *reinterpret_cast<const float4*>(row + i0)  // V % 4 == 0
+                                : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+        v[q][0] = w.x;
+        v[q][1] = w.y;
+        v[q][2] = w.z;
+        v[q][3] = w.w;
+      } else {
 #pragma unroll
-      for (int j = 0; j < kPer; ++j) {
-        const int i = base + t + 1024 * j;
-        v[j] = i < V ? row[i] : -INFINITY;
+        for (uint32_t j = 0; j < 4; ++j) v[q][j] = i0 + 1024 * j < V ? row[i0 + 1024 * j] : -INFINITY;
       }
     }
-    // ids ascend with j, so the first of equal values is kept
+    // ids ascend with q and j, so the first of equal values is kept
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int i = base + (kVec4 ? 4 * (t + 1024 * (j >> 2)) + (j & 3) : t + 1024 * j);
-      const bool take = (at < 0) | (!(v[j] <= best) & (best == best));
-      if (take & (i < V)) {
-        best = v[j];
-        at = i;
+    for (uint32_t q = 0; q < kGroups; ++q) {
+      if (base + q * kGroup >= V) continue;
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) {
+        const uint32_t i = base + q * kGroup + (kVec4 ? 4 * t + j : t + 1024 * j);
+        const bool take = !any | (!(v[q][j] <= best) & (best == best));
+        if (take & (i < V)) {
+          best = v[q][j];
+          at = i;
+          any = true;
+        }
       }
     }
   }
-  uint64_t key = at >= 0 ? value_index_key(best, static_cast<uint32_t>(at)) : 0ull;
+  uint64_t key = any ? value_index_key(best, at) : 0ull;
   key = wave_max_u64(key);
   if ((t & 63) == 0) part[t >> 6] = key;
   __syncthreads();

@@ -240,3 +240,9 @@ def test_argmax_first_and_nan(V):
     x[5] = float("nan")
     x[6, V // 2] = float("inf")
     assert np.array_equal(ops().argmax(x.cuda()).cpu().numpy(), np.argmax(x.numpy(), axis=1))
+
+
+# rows that end on and next to a group of 4096 ids, in the first and in a later pass
+@pytest.mark.parametrize("V", [4096, 4100, 8191, 28676, 32771, 36864])
+def test_argmax_row_ends(V):
+    test_argmax_first_and_nan(V)

@@ -260,6 +260,8 @@ __device__ __forceinline__ void topk_row(float* srow, int n, int k, int lane, fl
 // the result: one 16-byte LDS store), four tiles' rows requested together.
 // Candidates and visibility: the memory rules of the kernel below.
 constexpr int kTopkSmall = 1024;  // most entries of this kernel
+// Most workgroups of 1024 threads in a launch: its work-items are counted in 32 bits.
+constexpr int64_t kMaxGroups1024 = (1ll << 22) - 1;
 
 template <int NS>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void
@@ -1482,7 +1484,10 @@ extern "C" int32_t llmy_cmp_memory_prefill_bf16(
   float* wl = static_cast<float*>(workspace);
   int32_t* il = top_k > 0 ? reinterpret_cast<int32_t*>(wl + queries * H * Kmax) : nullptr;
   const size_t lds = static_cast<size_t>(rows) * (ncp + 1) * 4;
-  if (top_k > 0 && (head_dim == 64 || head_dim == 128) && n_entries <= kTopkSmall)
+  // past the 16-query grid's limit (some 67M query-heads) the 32-query kernel, whose
+  // grid is half as large, takes the call
+  if (top_k > 0 && (head_dim == 64 || head_dim == 128) && n_entries <= kTopkSmall &&
+      static_cast<int64_t>(B) * ((T + 15) / 16) * H <= kMaxGroups1024)
     topk_prefill_launch(B, s, q, q_ld, mk, mk_ld, T, n_entries, H, head_dim, slots_window, ratio,
                         top_k, scale * kLog2eC, wl, il);
   else if (top_k > 0)

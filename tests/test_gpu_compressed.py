@@ -113,6 +113,20 @@ def test_memory_prefill_topk_blocks(B, T, ratio, H, Dh, top_k):
     test_memory_prefill(B, T, ratio, H, Dh, 64, top_k)
 
 
+def test_memory_prefill_topk_more_blocks_than_a_launch_takes():
+    """2^22 blocks of 16 queries (17-token rows, 16 heads) are one more than a launch
+    of 1024-thread workgroups takes: the call runs on 32-query blocks.  One summary,
+    seen by each row's last token alone: that token's output is the summary."""
+    from hybrid_llm_amd import ops
+    B, T, H, Dh, Dv = 1 << 17, 17, 16, 64, 64
+    q = torch.zeros(B * T, H * Dh, dtype=torch.bfloat16, device="cuda")
+    mk = torch.zeros(B, H * Dh, dtype=torch.bfloat16, device="cuda")
+    mv = torch.randn(B, Dv, device="cuda").to(torch.bfloat16)
+    out = ops.cmp_memory_prefill(q, mk, mv, B, T, T, H, Dh, 1).view(B, T, Dv)
+    assert torch.equal(out[:, -1], mv)
+    assert not out[:, :-1].any()
+
+
 @pytest.mark.parametrize("T,ratio,top_k,levels", [(2048, 4, 32, 3), (2048, 4, 16, 9), (1024, 2, 5, 2)])
 def test_memory_prefill_topk_ties(T, ratio, top_k, levels):
     """Scores drawn from a few levels, so many summaries tie at the top-k

@@ -416,37 +416,51 @@ int32_t launch_tiles(const TileArgs& g, long long items, hipStream_t s) {
 int32_t dense_narrow_ws(const uint16_t* x, const uint16_t* w, void* out, const float* aux, int M,
                         int N, int K, int ldo, int epi, bool packed, hipStream_t s);
 
-// Tile shapes and the time of one round of them over the chip, in rounds of
-// single 128 x 128 tiles (us at K = 1024, bf16 out, packed weights: 11.7 for 256
-// tiles of 128 x 128, 16.7 of 128 x 192, 19.6 for 240 of 128 x 256, 28.8 for 256
-// of 256 x 192, 34.3 of 256 x 256).
+// Tile shapes and the time of one round of them (us, packed weights, bf16 out; K 256
+// to 4096): on an idle chip (at most 64 tiles) and on a full one (230 to 256), each
+// a fixed part and one per k.
 struct TileShape {
   int bm, bn;
-  float round;
+  float idle, idle_k, full, full_k;
 };
-constexpr TileShape kTileShapes[] = {
-    {128, 128, 1.f}, {128, 192, 1.43f}, {128, 256, 1.68f}, {256, 192, 2.46f}, {256, 256, 2.93f}};
+constexpr TileShape kTileShapes[] = {{128, 128, 3.6f, 0.0060f, 4.0f, 0.0082f},
+                                     {128, 192, 4.5f, 0.0074f, 5.5f, 0.0105f},
+                                     {128, 256, 5.0f, 0.0088f, 6.2f, 0.0131f},
+                                     {256, 192, 6.1f, 0.0120f, 7.0f, 0.0190f},
+                                     {256, 256, 7.1f, 0.0151f, 8.4f, 0.0243f}};
 
-// Modelled time of out[M, N] with a shape: whole rounds of workgroups (a second
-// 128 x 128 tile per CU shares the CU with the first: 384 tiles took 18.6 us, 480
-// 21.4, 768 33.9 against 11.7 for 256).
-float tile_cost(int shape, int M, int N) {
+// Modelled time (us) of out[M, N] with a shape: full rounds of workgroups and a last
+// one between the idle and the full chip's time by the square of its share of the
+// CUs.  A 128 x 128 tile starts beside another on its CU, which hides 2.5 us of each
+// further round.  Over 184 calls of 256 to 8192 rows, 16 to 6400 columns and K 256 to
+// 4096 the shape (and tail) chosen takes 0.14% more than the best one on average and
+// 7% at most (whole rounds at K = 1024's proportions: 0.65% and 24%).
+float tile_cost(int shape, int M, int N, int K) {
   const TileShape& t = kTileShapes[shape];
   const long long tiles = static_cast<long long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-  const float rounds = static_cast<float>((tiles + compute_units() - 1) / compute_units());
-  return shape == 0 ? 0.15f + 0.85f * rounds : t.round * rounds;
+  const int cus = compute_units();
+  const long long rounds = (tiles + cus - 1) / cus;
+  const float idle = t.idle + t.idle_k * K, full = t.full + t.full_k * K;
+  const float part = static_cast<float>(tiles - (rounds - 1) * cus) / cus;
+  return static_cast<float>(rounds - 1) * (full - (shape == 0 ? 2.5f : 0.f)) + idle +
+         (full - idle) * part * part;
 }
+
+// Modelled time (us) of the narrow launch that takes a column tail: its own, and
+// reading x again.
+float tail_cost(int M, int K) { return 3.5f + 3.2e-7f * static_cast<float>(M) * K; }
 
 // Rows below which outputs are summed in 256-wide blocks of k (tiles of 128 rows
 // only: the second set of sums takes registers that the larger ones do not have).
 constexpr int kBlockSumRows = 256;
 
 // The cheapest shape.  Every shape that a row count allows sums each output over k
-// in the same order, so the results do not depend on the choice.
-int tile_shape(int M, int N) {
+// in the same order, so the results do not depend on it (those of a column tail
+// depend on whether it is split off, below).
+int tile_shape(int M, int N, int K) {
   int best = 0;
   for (int i = 1; i < (M < kBlockSumRows ? 3 : 5); ++i)
-    if (tile_cost(i, M, N) < tile_cost(best, M, N)) best = i;
+    if (tile_cost(i, M, N, K) < tile_cost(best, M, N, K)) best = i;
   return best;
 }
 
@@ -469,16 +483,18 @@ int32_t dense_gemm_mfma(const uint16_t* x, const uint16_t* w, void* out, const f
   g.N = N;
   g.packed = packed;
   g.group_m = 4;
-  int shape = tile_shape(M, N);
+  int shape = tile_shape(M, N, K);
   // A narrow column tail (N = 256 n + 16 .. 64, e.g. a 4096-row projection
   // plus its 16 gate rows) can cost a whole column of tiles, often another
   // round of workgroups: then the whole columns run first and the tail columns
   // follow on the weight-streaming kernel with the rows split 16 per workgroup
-  // (the same output rows, column offset and stride N; about 5 us).
+  // (the same output rows, column offset and stride N), which sums them in
+  // 256-wide blocks of k.  us, split / one launch: 4096 x 4112 x 1024 37.9 / 40.2,
+  // 2048 x 4112 x 1024 24.1 / 21.8, 2048 x 4112 x 256 13.8 / 11.2.
   const int tail = N > 256 ? N % 256 : 0;
   if (tail > 0 && tail <= 64) {
-    const int whole = tile_shape(M, N - tail);
-    if (tile_cost(whole, M, N - tail) + 0.45f < tile_cost(shape, M, N)) {
+    const int whole = tile_shape(M, N - tail, K);
+    if (tile_cost(whole, M, N - tail, K) + tail_cost(M, K) < tile_cost(shape, M, N, K)) {
       g.N = N - tail;
       shape = whole;
     }

@@ -75,8 +75,9 @@ def test_linear_epilogues(M, N, K, epi, layout):
 
 # Rows from which the tiles take over, and one size per tile shape (128 x 128, 128
 # x 192, 128 x 256, 256 x 192, 256 x 256) with partial tiles in both directions.
-# Tolerances: fp32 sums of K products |x w| ~ 0.016 in another order (K 2^-24 K
-# 0.016 < 1e-5 at K = 512).
+# Tolerance: an output is a chain of K / 16 <= 32 MFMA steps, each of which rounds a
+# partial sum of at most some 2.5 (5.6 standard deviations of 0.02 sqrt(512)): 32 x 2.5 x
+# 2^-24 = 4.8e-6, and the residual's sum is one more rounding, relative to its own size.
 @pytest.mark.parametrize("M,N,K", [(95, 1040, 512), (96, 1040, 512), (97, 48, 256),
                                    (129, 3088, 256), (2030, 3040, 256), (2500, 3056, 256),
                                    (4090, 3040, 256), (4001, 3984, 512), (2048, 4112, 256)])
@@ -104,6 +105,13 @@ def test_linear_tile_shapes(M, N, K, epi):
         else:
             assert float((err - expect.abs() * 2.0 ** -23).max()) <= 1e-5
         assert bool((buf[M:] == 7.0).all())
+
+
+# column tails that run on the streaming kernel, beside tiles of both sums
+@pytest.mark.parametrize("M,N,K", [(4090, 4144, 256), (4090, 4112, 512), (200, 32784, 512)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+def test_linear_column_tails(M, N, K, epi):
+    test_linear_tile_shapes(M, N, K, epi)
 
 
 # The tiles take over from the streaming kernel at 96 rows; below 256 rows (and up to

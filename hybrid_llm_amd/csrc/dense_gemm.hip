@@ -197,12 +197,13 @@ __device__ __forceinline__ void tile_store(const TileArgs& a, const f32x16 (&acc
 //
 // Measured (us, K = 1024, packed weights, bf16 out, three operand sets in turn;
 // before: reads and copies in bursts, every output stored as its lane holds it):
-// 4096 x 3072: 44.0 -> 28.8 (894 TFLOP/s; 256 x 192 tiles, where 128 x 128 ones
-// ran 1.5 rounds), 4096 x 4096: 45.6 -> 34.3, 2048 x 3072: 28.1 -> 16.7, 4096 x
-// 1024: 16.9 -> 11.7, gated residual 24.6 -> 19.6.  The steady loop keeps the
-// matrix cores 84% busy (K 1024 -> 2048 adds 13.5 us to a 256 x 192 tile, its
-// MFMAs alone 11.4); the rest of a call is its first loads, the epilogue and the
-// launch, about 8 us.
+// 4096 x 3072: 44.2 -> 27.7 (930 TFLOP/s; 256 x 192 tiles, where 128 x 128 ones
+// ran 1.5 rounds), 4096 x 4096: 44.1 -> 33.7, 2048 x 3072: 26.4 -> 15.3, 4096 x
+// 1024: 16.0 -> 11.2, gated residual 23.1 -> 17.3.  A further 1024 of K take a 256 x
+// 192 tile 12.3 us on an idle chip (its MFMAs alone 10.2 at 2.4 GHz) and 19 on a full
+// one: 1.36 PFLOP/s, where power holds the clock (loops of MFMAs alone on random
+// operands reach 1.44 to 1.53).  The rest of a call is its first loads, the epilogue
+// and the launch, about 8 us.
 template <int N>
 __device__ __forceinline__ void settle_frags(u32x4 (&f)[N]) {
   static_assert(N >= 4 && N <= 8, "fragments");

@@ -93,7 +93,7 @@ __device__ __forceinline__ f32x4 mfma16_f32(const f32x4& a, const f32x4& b, f32x
 // is a chain of fp32 MFMAs whose operands are all lane-local, and T_ij^T in D
 // form is T in the scan's operand form.  Bound by reading K and writing T and
 // the factors (16 + 13.5 KiB per chunk and head of 128): 8 x 4096 tokens, 16
-// heads of 128: 46 us, 5.2 TB/s (a four-wave workgroup per chunk with the
+// heads of 128: 46 us, 5.5 TB/s (a four-wave workgroup per chunk with the
 // inverse in LDS: 108 us).
 template <int D>
 __global__ __launch_bounds__(64) void gdn_chunk_prep_kernel(
@@ -261,13 +261,16 @@ __global__ __launch_bounds__(64) void gdn_chunk_prep_kernel(
 // compiler would put every read next to its use and wait out some forty LDS
 // latencies a chunk.
 // The 16-byte chunks of K, Q and V rows are XOR-swizzled by row (on the source
-// side of the copies): row fragments (16-byte reads of 16 rows) are
-// conflict-free, and so are K^T's (ds_read_b64_tr_b16 of 8 rows).
+// side of the copies): by the bank map row fragments (16-byte reads of 16 rows)
+// meet no conflict, nor do K^T's (ds_read_b64_tr_b16 of 8 rows); the counter still
+// shows conflicts in 10% of the cycles, from reads not yet told apart.
 // Slices of one (b, h) run on one XCD (block id mod 8) and share its L2.
-// 8 x 4096 tokens, 16 heads of 128: 218 us, about 7.1k cycles a chunk (eight
-// equal waves that passed S, Y and U through LDS: 275 us, 9.2k).  No unit is
-// saturated (LDS active 45%, VALU 41%, matrix cores 33% of the cycles, HBM 3.6
-// TB/s): the recurrence's dependent products and the two barriers set the pace.
+// 8 x 4096 tokens, 16 heads of 128: 212 us of back-to-back calls (first calls on an
+// idle GPU up to 285), about 7.6k cycles a chunk (eight equal waves that passed S, Y
+// and U through LDS: 275 us, 9.2k).  No unit is saturated (LDS active 42% of the
+// cycles, VALU 37%, matrix cores 30%; 667 MB of HBM traffic, 3.1 TB/s): the
+// recurrence's dependent products, the reads in front of them and the two barriers
+// set the pace.
 template <int D>
 __device__ __forceinline__ int kq_swz(int t) {
   return D == 128 ? (4 * (t & 3)) | ((t >> 2) & 3) : (4 * ((t >> 1) & 1)) | ((t >> 2) & 3);

@@ -76,9 +76,10 @@ int32_t llmy_moe_permute(const int32_t* expert_ids, int32_t n_routes,
  * the slices in order (llmy_moe_route_decode).
  * weight_layout 0: W row-major [N,K] (nn.Linear); 1: W in the packed tile
  * order of llmy_pack_weights_bf16.  Limits: N % 16 == 0, K % 256 == 0.
- * M < 96 (decode batches): weight-streaming kernels; M >= 96 (prefill
- * sequences) with a 16-byte aligned out: MFMA tiles (128 x 128 to 256 x 256 per
- * workgroup).
+ * M < 96: weight-streaming kernels; M >= 96 with a 16-byte aligned out and
+ * operands below 2 GiB: MFMA tiles (128 x 128 to 256 x 256 per workgroup).  For
+ * K <= 2048 a row's result does not depend on M up to 255 rows (but for packed
+ * weights of N >= 8192 up to 64 rows, whose sums run over all of K in one chain).
  * Replaces linear_forward / k_linear_gemv (llmy_cuda/src/model.cpp:1467-1515)
  * and nn.Linear on the decode and prefill paths. */
 int32_t llmy_linear_bf16(const llmy_bf16* x, const llmy_bf16* w, void* out,

@@ -444,32 +444,32 @@ __device__ __forceinline__ bool fast_top_p(const float* x, uint32_t live, NucRow
                                            float top_p, float u, FastLds& fs, int* out_id) {
   const int t = threadIdx.x;
   const float depth = kFastDepth * r.b;
-  const int cut = depth < static_cast<float>(kFastBins - 1) ? static_cast<int>(depth) : kFastBins;
+  // buckets cut .. kFastBins - 1 are collected; the last one always is: the ids past
+  // the row are there
+  const int cut =
+      depth < static_cast<float>(kFastBins - 1) ? static_cast<int>(depth) : kFastBins - 1;
   for (int i = t; i < kFastBins; i += kNucThreads) fs.mass[i] = 0ull;
   __syncthreads();
   u64 deep = 0ull;
 #pragma unroll
   for (int j = 0; j < kNucPer; ++j) {
     const float xj = nuc_x(x, j);
-    const u64 w = nuc_weight<false>(xj, live, j, r);
-    if (w == 0ull) continue;  // ids outside the row among them: no atomics for nothing
+    const u64 w = nuc_weight<false>(xj, live, j, r);  // 0 for ids outside the row
     const int bin = fast_bin(xj, r);
     if (bin < cut)
       atomicAdd(&fs.mass[bin], w);
     else
       deep += w;
   }
-  if (cut < kFastBins) {  // uniform
 #pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) deep += __shfl_xor(deep, off, kWave);
-    if ((t & (kWave - 1)) == 0) atomicAdd(&fs.mass[kFastBins - 1], deep);
-  }
+  for (int off = 1; off < kWave; off <<= 1) deep += __shfl_xor(deep, off, kWave);
+  if ((t & (kWave - 1)) == 0) atomicAdd(&fs.mass[kFastBins - 1], deep);
   __syncthreads();
   u64 h0 = fs.mass[2 * t], h1 = fs.mass[2 * t + 1];
   u64 total;
   u64 P = nuc_excl_scan(h0 + h1, fs.wave_tot, &total);
   if (total == 0ull) return false;
-  bool whole = cut == kFastBins;
+  bool whole = cut == kFastBins - 1;
   // the bucket holding running mass thr, after the second pass if it is the
   // collected one
   auto find = [&](u64 thr) {

@@ -291,7 +291,9 @@ __device__ __forceinline__ int v_swz(int t) {
 // readfirstlane, or a v_readlane that restores a spilled SGPR).  m0 is reserved
 // (nothing is allocated to it, hence the compiler's warning), but the compiler
 // itself keeps values there for LDS-DMA builtins and indexed moves: the clobber
-// tells it that they are gone.
+// tells it that they are gone.  (The wait states cost 0.4 us of 34.6 at 1 x 1003 tokens,
+// 16 heads of 64, and nothing measurable at 128; one wait for several copies in one
+// statement was no faster.)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void lds_copy16(const u32x4& rsrc, uint32_t off, uint32_t dst) {

@@ -432,8 +432,8 @@ __device__ __forceinline__ bool fast_resolve(const float* x, uint32_t live, NucR
 // pass; masses are integers, so the picks are the same either way.
 // us at 64 rows, T = 0.8, p = 0.9, three sets of logits in turn, before (ids in
 // thread order, one atomic per id, every id's bucket formed in each resolve) -> now:
-// 32000 logits of spread 0.64 29.5 -> 24.1, 3 24.2 -> 18.6, 8 44.0 -> 17.9; 8192 of
-// spread 3 37.0 -> 16.6.
+// 32000 logits of spread 0.64 29.5 -> 24.1, 3 24.2 -> 18.3, 8 44.0 -> 17.7; 8192 of
+// spread 3 37.0 -> 17.6.
 constexpr float kFastDepth = 14.f;
 
 // The whole draw without top-k; false (uniformly) when a bucket overflows or

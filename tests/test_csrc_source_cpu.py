@@ -2,8 +2,9 @@
 
 The compiler treats an asm statement as one opaque instruction.  A register it writes
 must be named as clobbered, and the wait states that the hardware asks for between its
-operands' writers and its own memory instruction must be inside it.  An entry point may be called by any thread, so a value that a
-function keeps is initialised where it is declared.
+operands' writers and its own memory instruction must be inside it.  An entry point may
+be called by any thread, so a value that a function keeps is initialised where it is
+declared.
 """
 import re
 from pathlib import Path
